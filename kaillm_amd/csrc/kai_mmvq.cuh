@@ -322,6 +322,15 @@ __device__ __forceinline__ void mmvq_part(const uint8_t *__restrict__ weight, in
     }
 }
 
+template <int TYPE, int M, bool TWO_PASS, int DEPTH, int G, int RS, int KS = 1>
+__global__ __launch_bounds__((mmvq_threads<M, RS, G, KS>()))
+void mmvq_kernel(const uint8_t *__restrict__ weight, int64_t row_bytes, int nrows, int units_per_row,
+                 const block_q8_1 *__restrict__ y1, const block_q8_1 *__restrict__ y2, int y_row_blocks,
+                 const float *__restrict__ inverse, void *__restrict__ dst, int64_t stride_dst, int dst_bf16) {
+    mmvq_part<TYPE, M, TWO_PASS, DEPTH, G, RS, KS>(weight, row_bytes, nrows, units_per_row, y1, y2, y_row_blocks, inverse,
+                                                   dst, stride_dst, dst_bf16, blockIdx.x);
+}
+
 // The matrices of a launch: workgroups first[p] .. first[p + 1] take matrix p.
 struct MmvqArgs {
     const uint8_t *weight[GEMV_PARTS];
@@ -332,12 +341,14 @@ struct MmvqArgs {
 // One launch for the matrices of a merged projection that have one type: a decode launch of a
 // few thousand rows is 4 us of latency however few its bytes, and the matrices' waves fill the
 // chip together. Measured on MI355X in replayed graphs, with the preparation: Q4_0 2048 + 512 +
-// 512 rows of 2048 at four activation rows 21.1 -> 16 us (the kernels 13.3 -> 5.0).
+// 512 rows of 2048 at four activation rows 21.1 -> 16 us (the kernels 13.3 -> 5.0). A matrix by itself
+// has a kernel of its own: the choice of the matrix costs 0.1-0.25 us of a launch (with the
+// preparation, Q4_K 452 x 1792 at one row 5.9 -> 6.1 us, 34816 x 5120 20.8 -> 21.3 us).
 template <int TYPE, int M, bool TWO_PASS, int DEPTH, int G, int RS, int KS = 1>
 __global__ __launch_bounds__((mmvq_threads<M, RS, G, KS>()))
-void mmvq_kernel(MmvqArgs parts, int64_t row_bytes, int units_per_row, const block_q8_1 *__restrict__ y1,
-                 const block_q8_1 *__restrict__ y2, int y_row_blocks, const float *__restrict__ inverse,
-                 int64_t stride_dst, int dst_bf16) {
+void mmvq_group_kernel(MmvqArgs parts, int64_t row_bytes, int units_per_row, const block_q8_1 *__restrict__ y1,
+                       const block_q8_1 *__restrict__ y2, int y_row_blocks, const float *__restrict__ inverse,
+                       int64_t stride_dst, int dst_bf16) {
     const uint8_t *weight = parts.weight[0];
     void *dst = parts.dst[0];
     int nrows = parts.nrows[0], first = 0;
@@ -434,12 +445,25 @@ static void launch_sets(const GemvParts &w, int64_t k, const block_q8_1 *y1, con
         blocks += (w.n[p] + rows_per_block - 1) / rows_per_block;
     }
     if (blocks >= INT_MAX) throw Error("Too many GEMV rows");
+    const int y_blocks = static_cast<int>(k / QK8_1), bf16 = dst_bf16 ? 1 : 0;
+    const dim3 grid(static_cast<unsigned>(blocks));
+    if constexpr (M <= 8) {  // groups are decode calls
+        if (w.count > 1) {
+            auto kernel = mmvq_group_kernel<TYPE, M, TWO_PASS, DEPTH, G, RS, KS>;
+            static DeviceFlags raised;  // per instantiation and device
+            raise_dynamic_lds(reinterpret_cast<const void *>(kernel), MMVQ_LDS_BUDGET - 4096, raised,
+                              "Cannot raise the GEMV dynamic LDS limit");
+            kernel<<<grid, dim3(THREADS), lds, stream>>>(args, row_bytes, units, y1, y2, y_blocks, inverse, stride_dst, bf16);
+            return;
+        }
+    }
+    if (w.count != 1) throw Error("One matrix to a GEMV of more than 8 rows");
     auto kernel = mmvq_kernel<TYPE, M, TWO_PASS, DEPTH, G, RS, KS>;
-    static DeviceFlags lds_raised;  // per instantiation and device
+    static DeviceFlags lds_raised;
     raise_dynamic_lds(reinterpret_cast<const void *>(kernel), MMVQ_LDS_BUDGET - 4096, lds_raised,
                       "Cannot raise the GEMV dynamic LDS limit");
-    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(THREADS), lds, stream>>>(
-        args, row_bytes, units, y1, y2, static_cast<int>(k / QK8_1), inverse, stride_dst, dst_bf16 ? 1 : 0);
+    kernel<<<grid, dim3(THREADS), lds, stream>>>(w.weight[0], row_bytes, args.nrows[0], units, y1, y2, y_blocks, inverse,
+                                                 w.dst[0], stride_dst, bf16);
 }
 
 template <int TYPE, int M, bool TWO_PASS, int G>
