@@ -476,7 +476,22 @@ static void launch_variant(const GemvParts &w, int64_t n, int64_t k, const block
                 return;
             }
         }
-        switch (gemv_k_split<TYPE, M>(n, k, G, device_cu_count())) {
+        const int ks = gemv_k_split<TYPE, M>(n, k, G, device_cu_count());
+        if constexpr (M > 4) {
+            // a matrix that alone is split more finely keeps its 512 threads to a staged activation
+            // (128 unsplit; Q4_0 12 + 4164 + 3216 rows of 14208 at five activation rows 142 -> 115 us)
+            bool finer = false;
+            for (int p = 0; p < w.count; ++p) finer |= gemv_k_split<TYPE, M>(w.n[p], k, G, device_cu_count()) > ks;
+            if (w.count > 1 && finer) {
+                for (int p = 0; p < w.count; ++p) {
+                    GemvParts one;
+                    one.add(w.weight[p], w.n[p], w.dst[p]);
+                    launch_variant<TYPE, M, TWO_PASS, G>(one, w.n[p], k, y1, y2, inverse, dst_bf16, stride_dst, stream);
+                }
+                return;
+            }
+        }
+        switch (ks) {
             case 4: launch_sets<TYPE, M, TWO_PASS, G, 1, 4>(w, k, y1, y2, inverse, dst_bf16, stride_dst, stream); return;
             case 2: launch_sets<TYPE, M, TWO_PASS, G, 1, 2>(w, k, y1, y2, inverse, dst_bf16, stride_dst, stream); return;
             default: break;
