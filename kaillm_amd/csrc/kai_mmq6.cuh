@@ -241,35 +241,6 @@ __global__ __launch_bounds__(64 * GN * GK) __attribute__((amdgpu_waves_per_eu(WP
     else mmqh_store<1, CT, GK>(out, mine, dst, stride_dst, inverse, m0, n0 + wrow0, m, n, kz, lane);
 }
 
-// Tile configurations: activation rows, weight rows, K groups (four waves two workgroups to a CU,
-// else eight waves to a CU).
-enum Mmq6Id : int { MMQ6_NONE = -1, MMQ6_96X128, MMQ6_96X128_2, MMQ6_96X64_4, MMQ6_64X64_4, MMQ6_IDS };
-// Which one an m-row product of an n x k matrix takes, or MMQ6_NONE: the int8 tile kernel
-// (kai_mmq.cuh), whose many small tiles are faster up to 80 rows and on matrices of few rows. Its
-// time is taken as the padded work at 184 TOP/s. Measured on MI355X (kernel alone, us; stage times
-// below from the same runs): 5120 x 17408 at 96 / 160 / 256 / 512 rows int8 tiles 114 / 232 / 262 / 412,
-// here 129 / 133 / 176 / 281; 5120 x 6144 at 96 / 160 rows 42 / 84, here 52 / 55; 34816 x 5120 at 64 / 96
-// rows 134 / 251, here 154 / 163; 512 x 5120 at 160 / 1000 rows 15 / 40, here 39 / 41.
-inline Mmq6Id mmq6_plan(int64_t n, int64_t k, int64_t m) {
-    struct Config {
-        int bm, bn, slots;
-        double low, high;  // us of a stage, up to one workgroup per CU and with two
-    };
-    constexpr Config CONFIGS[MMQ6_IDS] = {{96, 128, 512, 1.22, 1.80}, {96, 128, 256, 1.03, 1.16}, {96, 64, 256, 0.60, 0.65},
-                                          {64, 64, 256, 0.48, 0.50}};
-    if (m <= 80) return MMQ6_NONE;
-    const double stages = double(k) / 64, padded = double((m + 63) / 64 * 64);
-    double best = 2.0 * padded * double(n) * double(k) / 184e6;
-    Mmq6Id id = MMQ6_NONE;
-    for (int c = 0; c < MMQ6_IDS; ++c) {
-        const Config &f = CONFIGS[c];
-        const int64_t wgs = (n + f.bn - 1) / f.bn * ((m + f.bm - 1) / f.bm), rem = wgs % f.slots;
-        const double us = double(wgs / f.slots) * (6.0 + stages * f.high) +
-                          (rem ? 6.0 + stages * (rem <= 256 && f.slots > 256 ? f.low : f.high) : 0.0);
-        if (us < best) best = us, id = Mmq6Id(c);
-    }
-    return id;
-}
 // The product on its plan's configuration; false: the int8 tile kernel is to take it.
 bool launch_mmq6(const void *weight, int64_t n, int64_t k, int64_t m, const uint8_t *plane, const float *inverse, void *dst,
                  bool dst_bf16, int64_t stride_dst, hipStream_t stream);
