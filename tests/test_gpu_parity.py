@@ -15,6 +15,7 @@ import pytest
 import torch
 
 import _oracle as O
+import _plan as P
 
 pytestmark = pytest.mark.gpu
 
@@ -631,19 +632,18 @@ def test_batched_prefill_tiles(kai, qtype, weights, m, n, k):
 
 # More tiles than CUs with a short last round: the tiles of a rectangle at the output's end run
 # in K pieces whose sums a second kernel adds into that rectangle, in place of an unsplit plan's
-# short round or a K split's extra rounds; the other tiles run whole. Rectangles (rows r0.., weight
-# rows c0..): Q4_K on 256 x 128 tiles, 2 x 141 tiles, the last 26 in 4 pieces of one 256-value
-# step (the last tile 80 wide); Q4_0 at 40 rows on 128 x 96 tiles and IQ3_S and Q2_K at 120 rows
-# on 128 x 128 tiles, 258 tiles, the last 2 (232 columns, the last tile 104 wide) in 4 pieces
-# over every row; two activation tiles high: Q4_K and Q2_K, 14 x 20 tiles of 256 x 128, the last
-# 12 of the last 2 (412 rows, the last tile 68 wide) in 2 pieces.
-TAIL = [(O.Q4_K, 300, 18000, 1024, 256, 14720), (O.Q4_0, 40, 33000, 1024, 0, 32768),
-        (O.IQ3_S, 120, 33000, 1024, 0, 32768), (O.Q2_K, 120, 33000, 1024, 0, 32768),
-        (O.Q4_K, 3484, 2500, 512, 3072, 1024), (O.Q2_K, 3484, 2500, 512, 3072, 1024)]
+# short round or a K split's extra rounds; the other tiles run whole. One of each kind, the plan
+# asked: rectangles over every activation row (r0 = 0) and from an activation tile on with whole
+# tiles beside them, on tiles of 64, 96, 128 and 128 x 128 rows with two K groups.
+TAIL = [(O.Q4_K, 802, 9644, 1792), (O.Q4_0, 44, 32872, 800), (O.IQ3_S, 120, 32968, 1792), (O.Q2_K, 878, 9352, 1280),
+        (O.Q4_0, 897, 8388, 1376), (O.Q8_0, 1052, 3944, 1120), (O.IQ3_S, 159, 17224, 2816)]
 
 
-@pytest.mark.parametrize("qtype,m,n,k,r0,c0", TAIL, ids=[f"{O.NAMES[t]}-{m}x{n}x{k}" for t, m, n, k, _, _ in TAIL])
-def test_batched_tail_tiles_in_k_pieces(kai, qtype, m, n, k, r0, c0):
+@pytest.mark.parametrize("qtype,m,n,k", TAIL, ids=[f"{O.NAMES[t]}-{m}x{n}x{k}" for t, m, n, k in TAIL])
+def test_batched_tail_tiles_in_k_pieces(kai, qtype, m, n, k):
+    plan = P.folded(qtype, n, k, m)
+    assert plan.pieces > 1 and plan.c0 > 0 and (plan.r0 > 0) == (m > 128), plan
+    r0, c0 = plan.r0, plan.c0
     print(f"batched tail tiles {O.NAMES[qtype]} m={m} n={n} k={k}", flush=True)
     rng = np.random.default_rng(qtype + m)
     w = O.random_blocks(qtype, n, k, rng)
@@ -673,6 +673,8 @@ def test_batched_tail_in_a_group_with_unaligned_columns(kai):
     print("batched tail in an unaligned group", flush=True)
     rng = np.random.default_rng(33002)
     m, k = 40, 1024
+    plan = P.folded(O.Q4_0, 33002, k, m)
+    assert plan.pieces > 1 and (plan.c0, plan.cols) == (32768, 234), plan
     w1 = O.random_blocks(O.Q4_0, 33002, k, rng)
     w2 = O.random_blocks(O.Q4_0, 2, k, rng)
     mats = [(O.Q4_0, w1, to_dev(w1)), (O.Q4_0, w2, to_dev(w2))]
