@@ -109,6 +109,8 @@ def kernel_name(qtype, m, n, k):
     if m > 16:
         if qtype in (Q4_K, Q4_0, Q8_0, IQ3_S, Q2_K):  # kai_launch.h mmq_uses_h
             return "fp16 folded-operand GEMM (kai_fused_mmq_run: fp16 image + mmqh_kernel)"
+        if m > 80:  # kai_batched_plan.h mmq6_plan
+            return "Q6_K GEMM (kai_fused_mmq_run: GGML MMQ planes + mmq6_kernel, or mmq_kernel on few rows)"
         return "int8 MMQ (kai_fused_mmq_run: GGML MMQ planes + mmq_kernel)"
     if m > 8:
         if persistent(n, image=True):

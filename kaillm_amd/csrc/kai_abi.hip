@@ -126,7 +126,8 @@ void run_mmq_group(const void *const *weights, const int *types, const int64_t *
     for (int i = 0; i < count; ++i) {
         const int l = kai::mmq_layout(types[i]);
         char *out = static_cast<char *>(dst) + col * elem;
-        if (i % kai::DECODE_PARTS == 0 && i + 1 < count && m <= kai::MMQS_MAX_ROWS) {  // up to four in one launch
+        // up to four in one launch, in fixed windows: one that the launch refuses goes matrix by matrix
+        if (i % kai::DECODE_PARTS == 0 && i + 1 < count && m <= kai::MMQS_MAX_ROWS) {
             kai::DecodeParts parts;
             int64_t at = col;
             for (int j = i; j < count && parts.count < kai::DECODE_PARTS; at += rows[j++])

@@ -1,5 +1,6 @@
-// Batched GEMM of Q6_K for more than 16 activation rows, on fp16 MFMA with whole-number operands:
-// kai_fused_mmq_run's and the legacy op's product over the int8 activation plane.
+// Batched GEMM of Q6_K above 80 activation rows where its plan prefers it to the int8 tile kernel
+// (mmq6_plan), on fp16 MFMA with whole-number operands: kai_fused_mmq_run's and the legacy op's product
+// over the int8 activation plane.
 //
 // Arithmetic. Per 32-value block the reference takes the integer dot of the activation codes q with
 // the weight codes (c - 32) times their int8 scales (one per 16 values), times the activation scale
@@ -9,7 +10,7 @@
 // exact too, and every partial sum of a block is a whole number below 32 * 127 * 4096 < 2^24, so
 // four MFMAs leave the block's integer dot in fp32, exactly, with no conversion left to do:
 //   y += d * sum over the superblock's blocks of d8 * dot.
-// The int8 tile kernel this replaced above 16 rows spent 20 VALU instructions per int8 MFMA on the
+// The int8 tile kernel spends 20 VALU instructions per int8 MFMA on the
 // two scales' combination and conversion; here a 32 x 32 x 32 block takes 128 cycles of the matrix pipe
 // and about 40 VALU instructions (16 for d8, 2 for d, the rest the weights' and activation's share).
 // 5120 x 17408, kernel alone: 160 rows 232 -> 133 us, 512 rows 412 -> 281 us, 2048 rows 1270 -> 975 us.
