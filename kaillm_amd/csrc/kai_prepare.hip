@@ -820,6 +820,7 @@ __global__ __launch_bounds__(PRODUCE_THREADS) void produce_kernel(ProduceArgs p)
     Raw8<0> wraw[W_AHEAD ? RUNS : 1];
 #pragma unroll
     for (int i = 0; i < RUNS; ++i) {
+        if (PRODUCE_THREADS * i >= nruns) break;  // uniform
         const int c = 8 * min(t + PRODUCE_THREADS * i, nruns - 1);
         if constexpr (MODE == PRODUCE_VIEW)
             load_raw8<XT>(xr + ((c / p.s) % p.a) * p.b * p.s + (c / (p.a * p.s)) * p.s + c % p.s, raw[i]);
@@ -831,7 +832,10 @@ __global__ __launch_bounds__(PRODUCE_THREADS) void produce_kernel(ProduceArgs p)
         if (p.res) {
             const auto *rr = static_cast<const typename Src<RT>::T *>(p.res) + static_cast<int64_t>(row) * p.stride_r;
 #pragma unroll
-            for (int i = 0; i < RUNS; ++i) load_raw8<RT>(rr + 8 * min(t + PRODUCE_THREADS * i, nruns - 1), rraw[i]);
+            for (int i = 0; i < RUNS; ++i) {
+                if (PRODUCE_THREADS * i >= nruns) break;
+                load_raw8<RT>(rr + 8 * min(t + PRODUCE_THREADS * i, nruns - 1), rraw[i]);
+            }
         }
     }
     float v[RUNS][8];
