@@ -738,7 +738,7 @@ void launch_prepare_mmq(const void *x, int x_dtype, int64_t m, int64_t k, int64_
 //          the input dtype, silu(g) = g / (1 + exp(-g));
 //   norm   v = x (+ r, written to the fp32 residual stream), y = bf16(v * rstd * w32) with
 //          rstd = 1 / sqrt(sum(v^2) / k + eps); the activation quantises the stored y.
-// view and norm: one workgroup of PRODUCE_THREADS per row (swiglu: several, below); run r of 8
+// One workgroup of PRODUCE_THREADS per row (swiglu of long rows: several, below); run r of 8
 // values belongs to thread r % PRODUCE_THREADS, so the four runs of a 32-value block sit in one
 // quad. One workgroup's time is latency: every load of the row, the norm's weight too, is issued
 // before the first is used (RUNS runs per thread, clamped), one memory round trip instead of
@@ -778,7 +778,12 @@ __device__ __forceinline__ float round_to_src(float v) {
     else return v;
 }
 
-enum ProduceMode { PRODUCE_VIEW, PRODUCE_NORM };
+template <int DTYPE>
+__device__ __forceinline__ float swiglu_exact(float g, float u) {
+    return round_to_src<DTYPE>(round_to_src<DTYPE>(g / (1.0f + produce_expf(-g))) * u);
+}
+
+enum ProduceMode { PRODUCE_VIEW, PRODUCE_SWIGLU, PRODUCE_NORM };
 
 struct ProduceArgs {
     const void *x;  // view: x; swiglu: [gate | up]; norm: x
@@ -826,6 +831,7 @@ __global__ __launch_bounds__(PRODUCE_THREADS) void produce_kernel(ProduceArgs p)
             load_raw8<XT>(xr + ((c / p.s) % p.a) * p.b * p.s + (c / (p.a * p.s)) * p.s + c % p.s, raw[i]);
         else
             load_raw8<XT>(xr + c, raw[i]);
+        if constexpr (MODE == PRODUCE_SWIGLU) load_raw8<RT>(xr + k + c, rraw[i]);  // RT is XT
         if constexpr (W_AHEAD) load_raw8<0>(p.w32 + c, wraw[i]);
     }
     if constexpr (MODE == PRODUCE_NORM) {
@@ -858,6 +864,12 @@ __global__ __launch_bounds__(PRODUCE_THREADS) void produce_kernel(ProduceArgs p)
 #pragma unroll
             for (int j = 0; j < 8; ++j) ss = fmaf(v[i][j], v[i][j], ss);
         } else {
+            if constexpr (MODE == PRODUCE_SWIGLU) {
+                float u[8];
+                convert8<RT>(rraw[i], u);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[i][j] = swiglu_exact<XT>(v[i][j], u[j]);
+            }
 #pragma unroll
             for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
         }
@@ -905,7 +917,7 @@ static void launch_produce(const ProduceArgs &a, int64_t m, hipStream_t stream) 
     else produce_kernel<MODE, XT, RT, PRODUCE_RUNS><<<grid, block, 0, stream>>>(a);
 }
 
-// ---- swiglu. A row's exact silu and rounding are about 60 VALU instructions a value: one workgroup
+// ---- swiglu of more than SWIGLU_SHORT values. A row's exact silu and rounding are about 60 VALU instructions a value: one workgroup
 // per row spent 13.4 us on a row of 17408. The only value that joins the row's blocks is the
 // exponent of its maximum, so several workgroups share a row: each finds that exponent by
 // itself from estimates of all values (8 instructions, the hardware's exp2 and reciprocal) and
@@ -922,6 +934,8 @@ static void launch_produce(const ProduceArgs &a, int64_t m, hipStream_t stream) 
 // both maxima as they do of the exact one, infinities make A or b infinite. Else (2 % of rows, by
 // chance) the workgroup takes the exact maximum of every value whose estimate does not rule it out
 // (a >= (1 - 2 w) A, or bounded only).
+constexpr int SWIGLU_SHORT = 4096;  // one run a thread of one workgroup: 256 to 2048 values 3.4-4.0 us, several
+                                    // workgroups 4.1-4.6; 4096 3.8-4.5 / 4.2-4.6, 5120 5.0-6.1 / 4.2-4.6
 constexpr int SWIGLU_THREADS = 1024;
 constexpr int SWIGLU_RUNS = 4;  // k <= 32768
 constexpr int SWIGLU_OWN = 128;  // runs of a workgroup's blocks: two of its waves, one run each
@@ -929,10 +943,6 @@ template <int DTYPE> constexpr float swiglu_gate() { return DTYPE == 2 ? -12.0f 
 template <int DTYPE> constexpr float swiglu_low() { return DTYPE == 2 ? 0x1p-13f : 0x1p-120f; }
 template <int DTYPE> constexpr float swiglu_high() { return DTYPE == 2 ? 0x1p+15f : 0x1p+126f; }
 
-template <int DTYPE>
-__device__ __forceinline__ float swiglu_exact(float g, float u) {
-    return round_to_src<DTYPE>(round_to_src<DTYPE>(g / (1.0f + produce_expf(-g))) * u);
-}
 // the estimate, or 0 where bounded only (then b > 0 for u != 0)
 template <int DTYPE>
 __device__ __forceinline__ float swiglu_estimate(float g, float u, float &b) {
@@ -1047,6 +1057,16 @@ void launch_prepare_swiglu(const void *gate_up, int dtype, int64_t m, int64_t k,
     ProduceArgs p = produce_args(k, out);
     p.x = gate_up;
     p.stride_x = stride;
+    if (k <= SWIGLU_SHORT) {
+        static_assert(SWIGLU_SHORT <= 8 * PRODUCE_THREADS, "one run a thread");
+        const dim3 rows(static_cast<unsigned>(m)), threads(PRODUCE_THREADS);
+        switch (dtype) {
+            case 0: produce_kernel<PRODUCE_SWIGLU, 0, 0, 1><<<rows, threads, 0, stream>>>(p); return;
+            case 1: produce_kernel<PRODUCE_SWIGLU, 1, 1, 1><<<rows, threads, 0, stream>>>(p); return;
+            case 2: produce_kernel<PRODUCE_SWIGLU, 2, 2, 1><<<rows, threads, 0, stream>>>(p); return;
+            default: throw Error("Fused activations must be F32, BF16 or F16");
+        }
+    }
     const int64_t parts = (k / 8 + SWIGLU_OWN - 1) / SWIGLU_OWN;
     const dim3 grid(static_cast<unsigned>(m), static_cast<unsigned>(parts)), block(SWIGLU_THREADS);
     switch (dtype) {

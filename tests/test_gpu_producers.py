@@ -46,7 +46,7 @@ def test_view_bit_exact(kai, dtype, m, a, b, s, pad):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("m,k,pad", [(1, 256, 0), (3, 5120, 64), (8, 17408, 0), (2, 32768, 0), (4, 96, 32)])
+@pytest.mark.parametrize("m,k,pad", [(1, 256, 0), (3, 5120, 64), (8, 17408, 0), (2, 32768, 0), (4, 96, 32), (2, 4096, 0), (3, 4128, 32)])
 def test_swiglu_bit_exact(kai, dtype, m, k, pad):
     print(f"swiglu dtype={dtype} m={m} k={k} pad={pad}", flush=True)
     rng = np.random.default_rng(k * 3 + m)
@@ -65,7 +65,7 @@ def test_swiglu_bit_exact(kai, dtype, m, k, pad):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("k", [1024, 1056, 17408])
+@pytest.mark.parametrize("k", [1024, 1056, 4128, 17408])  # above 4096 on several workgroups a row
 def test_swiglu_row_exponent(kai, dtype, k):
     """Rows whose maximum an estimate cannot place: within a rounding or two of a power of two, subnormal,
     overflowing fp16, all gates negative, tiny or zero, the largest product under a tiny or a far negative gate."""
