@@ -478,11 +478,14 @@ static void launch_variant(const GemvParts &w, int64_t n, int64_t k, const block
         }
         const int ks = gemv_k_split<TYPE, M>(n, k, G, device_cu_count());
         if constexpr (M > 4) {
-            // a matrix that alone is split more finely keeps its 512 threads to a staged activation
-            // (128 unsplit; Q4_0 12 + 4164 + 3216 rows of 14208 at five activation rows 142 -> 115 us)
-            bool finer = false;
-            for (int p = 0; p < w.count; ++p) finer |= gemv_k_split<TYPE, M>(w.n[p], k, G, device_cu_count()) > ks;
-            if (w.count > 1 && finer) {
+            // An unsplit workgroup is 128 threads to a staged activation, a split one 512. Where fewer than
+            // three stagings fit a CU, matrices that alone are split keep launches of their own (Q4_0 at five
+            // rows, us together / apart: 12 + 4164 + 3216 rows of 14208 142 / 115, 1200 + 5000 + 2000 + 9000 of
+            // 12320 162 / 158, of 8224 62 / 68, of 3104 21 / 34; 12 + 2100 + 2000 of 8224, split in two
+            // together and in four apart, 18 / 29).
+            bool split = false;
+            for (int p = 0; p < w.count; ++p) split |= gemv_k_split<TYPE, M>(w.n[p], k, G, device_cu_count()) > 1;
+            if (w.count > 1 && ks == 1 && split && 3 * mmvq_act_lds_bytes(M, k, TWO_PASS) > size_t(MMVQ_LDS_BUDGET)) {
                 for (int p = 0; p < w.count; ++p) {
                     GemvParts one;
                     one.add(w.weight[p], w.n[p], w.dst[p]);
