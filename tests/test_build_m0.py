@@ -1,7 +1,9 @@
 """The folded GEMM's global-to-LDS copies set M0 in an asm statement, which is safe only while
 nothing else in those kernels uses M0 (the compiler does not know the statement changes it).
 This checks the built library's own gfx950 code: in every mmqh_kernel, each instruction that
-names M0 is an `s_mov_b32 m0, ...` directly followed by a `global_load_lds_dwordx4`."""
+names M0 is an `s_mov_b32 m0, ...` directly followed by one wait state (`s_nop`, which the hardware
+requires between a scalar write of M0 and a copy that reads it) and a `global_load_lds_dwordx4`; the copies
+of every other kernel, which the compiler emits, keep that wait state too."""
 import re
 import shutil
 import subprocess
@@ -32,12 +34,15 @@ def test_folded_gemm_m0_only_before_copies(tmp_path):
             if m:
                 current = m.group(1)
                 continue
+            if "global_load_lds" in line and re.match(r"s_\w+ m0,", text[i - 1].strip()):
+                other.append((current[:60], "no wait state"))
             if not current or "mmqh_kernel" not in current:
                 continue
             kernels.add(current)
             if re.search(r"\bm0\b", line):
                 ins = line.strip()
-                if ins.startswith("s_mov_b32 m0,") and i + 1 < len(text) and "global_load_lds_dwordx4" in text[i + 1]:
+                if (ins.startswith("s_mov_b32 m0,") and i + 2 < len(text) and text[i + 1].strip().startswith("s_nop")
+                        and "global_load_lds_dwordx4" in text[i + 2]):
                     writes += 1
                 else:
                     other.append((current[:60], ins))
